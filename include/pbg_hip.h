@@ -38,7 +38,8 @@ typedef enum pbg_status {
   PBG_ERR_INVALID = -1,     /* bad argument (shape, enum, null pointer) */
   PBG_ERR_WORKSPACE = -2,   /* workspace missing or too small */
   PBG_ERR_LAUNCH = -3,      /* HIP reported an error at launch */
-  PBG_ERR_UNSUPPORTED = -4  /* a combination this build does not implement */
+  PBG_ERR_UNSUPPORTED = -4, /* a combination this build does not implement */
+  PBG_ERR_INDEX = -5        /* an id outside its table (the calls that check ids) */
 } pbg_status;
 
 /* Names follow the reference's registries: OPERATORS / DYNAMIC_OPERATORS
@@ -196,8 +197,7 @@ typedef struct pbg_step_buffers {
    * [0, num_*_rows) (or [0, num_relations)) is clamped to the nearest valid one, so the
    * step reads and updates row 0 or the last row instead, where the reference's
    * F.embedding raises IndexError (model.py:60-61).  A caller that cannot vouch for
-   * its ids checks them first (pytorch_biggraph_amd.native.StepRunner.train(check_ids=True)
-   * does, with one device reduction per array). */
+   * its ids calls pbg_train_step_checked instead. */
   const int64_t* lhs;         /* [K, B] */
   const int64_t* rhs;         /* [K, B] */
   const int64_t* rel;         /* standard: [K]; dynamic: [K, B] */
@@ -246,6 +246,10 @@ int pbg_sample_uniform_negatives(uint64_t seed, int32_t side, int64_t num_rows, 
 
 size_t pbg_train_step_workspace_bytes(const pbg_step_desc* desc);
 int pbg_train_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, pbg_stream_t stream);
+/* The same step, or PBG_ERR_INDEX with tables, sums and parameters as they were if any id is outside what it
+ * indexes.  `bad`: one word of PINNED host memory, not shared with another call under way.  The host waits, inside
+ * the call, for the check of the ids (not for the step): not capturable into a graph. */
+int pbg_train_step_checked(const pbg_step_desc* desc, const pbg_step_buffers* bufs, int32_t* bad, pbg_stream_t stream);
 
 /* The same step with HIP events recorded on `stream` between its stages; waits
  * for the step to finish and writes the pbg_train_step_num_stages() stage
@@ -301,6 +305,16 @@ int pbg_model_forward(const pbg_step_desc* desc, const pbg_step_buffers* bufs, f
 int pbg_model_ranks(const pbg_step_desc* desc, const pbg_step_buffers* bufs, float* lhs_pos, float* rhs_pos,
                     int64_t* lhs_rank, int64_t* rhs_rank, float* loss_edge, int64_t auc_samples, uint64_t auc_seed,
                     int64_t* auc_hits, pbg_stream_t stream);
+
+/* What a ranking evaluation reports of those outputs (eval.py:57-81), over `count` edges, to PINNED host memory:
+ * out[0] = sum of loss_edge; then per side (lhs, rhs) 6 values: sum of ranks, sum of 1 / rank, ranks <= 1, <= 10,
+ * <= 50, auc_hits[side] (0 without auc_hits).  out[13] != 0: an id of the call `desc` / `bufs` describe is outside its
+ * table (the ranks are then those of clamped ids).  `scratch`: pbg_rank_sums_scratch_bytes() bytes of device memory.
+ * Everything is queued on `stream`; the caller waits for it before it reads `out` (14 doubles). */
+size_t pbg_rank_sums_scratch_bytes(void);
+int pbg_rank_sums(const pbg_step_desc* desc, const pbg_step_buffers* bufs, int64_t count, const int64_t* lhs_rank,
+                  const int64_t* rhs_rank, const float* loss_edge, const int64_t* auc_hits, double* out, void* scratch,
+                  pbg_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Plugin-level entry points: one operator / comparator / loss at a time, forward

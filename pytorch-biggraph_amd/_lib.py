@@ -19,6 +19,7 @@ PBG_ERR_INVALID = -1
 PBG_ERR_WORKSPACE = -2
 PBG_ERR_LAUNCH = -3
 PBG_ERR_UNSUPPORTED = -4
+PBG_ERR_INDEX = -5
 
 
 class StepDesc(ctypes.Structure):
@@ -92,12 +93,15 @@ SIGNATURES = {
     "pbg_sample_uniform_negatives": (c_int32, [c_uint64, c_int32, c_int64, c_int64, c_void_p, c_void_p]),
     "pbg_train_step_workspace_bytes": (c_size_t, [POINTER(StepDesc)]),
     "pbg_train_step": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_void_p]),
+    "pbg_train_step_checked": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_void_p, c_void_p]),
     "pbg_train_step_num_stages": (c_int32, []),
     "pbg_train_step_is_fused": (c_int32, [POINTER(StepDesc)]),
     "pbg_train_step_route": (c_int32, [POINTER(StepDesc)]),
     "pbg_train_step_profile": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_void_p, POINTER(c_float)]),
     "pbg_model_ranks": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int64, c_uint64, c_void_p, c_void_p]),
+    "pbg_rank_sums_scratch_bytes": (c_size_t, []),
+    "pbg_rank_sums": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_int64] + [c_void_p] * 7),
     "pbg_model_forward": (c_int32, [POINTER(StepDesc), POINTER(StepBuffers), c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_void_p]),
     "pbg_operator_forward": (c_int32, [c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
@@ -161,6 +165,8 @@ def check(status: int) -> None:
     msg = lib().pbg_last_error().decode("utf-8", "replace")
     if status == PBG_ERR_INVALID:
         raise ValueError(msg)
+    if status == PBG_ERR_INDEX:
+        raise IndexError(msg)
     if status == PBG_ERR_UNSUPPORTED:
         raise NotImplementedError(msg)
     raise PbgError(f"pbg status {status}: {msg}")

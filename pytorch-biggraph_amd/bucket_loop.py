@@ -32,7 +32,7 @@ from typing import Callable, Dict, List, Optional, Sequence, Tuple
 import torch
 
 from . import native
-from .eval import ranking_stats_from_ranks
+from .eval import ranking_stats_from_sums
 from .losses import LOSS_FUNCTIONS
 from .stats import Stats
 from .util import round_up_to_nearest_multiple
@@ -465,11 +465,10 @@ class BucketLoop:
             # ranks, loss (AbstractBatchProcessor.calc_loss, batching.py:139-150, with relation weights of 1) and the
             # AUC count per edge from one call; the [K, B, N] score tensors are never formed
             self.eval_calls += 1
-            _, _, lhs_rank, rhs_rank, loss_edge, hits = runner.ranks(l, r, t, ul, ur, auc_samples=count,
-                                                                     auc_seed=(self.seed << 20) + self.eval_calls)
-            sides = [s for s, off in ((0, runner.spec.disable_lhs_negs), (1, runner.spec.disable_rhs_negs)) if not off]
-            stats.append(ranking_stats_from_ranks([(lhs_rank, rhs_rank)[s] for s in sides], float(loss_edge.sum()), count,
-                                                  [hits[s] for s in sides], count))
+            loss, sides = runner.rank_sums(l, r, t, ul, ur, auc_samples=count, auc_seed=(self.seed << 20) + self.eval_calls,
+                                           check_ids=False)
+            off = (runner.spec.disable_lhs_negs, runner.spec.disable_rhs_negs)
+            stats.append(ranking_stats_from_sums([side for side, skip in zip(sides, off) if not skip], loss, count, count))
         return Stats.sum(stats)
 
     def _train_bucket(self, b: Bucket, tables) -> BucketStats:

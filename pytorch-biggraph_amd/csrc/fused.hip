@@ -24,6 +24,12 @@ namespace pbg {
 namespace {
 
 
+// A call that checks its ids (c.id_bad): an entity id of this chunk, or its batch's relation, is outside what it
+// indexes.  The threads that fetch the ids look at them on the way; slots past the operand rows repeat ids of the batch.
+__device__ __forceinline__ void fused_check_id(const StepCtx& c, const SideCtx& sd, int k, int64_t id) {
+  if (c.id_bad && ((uint64_t)id >= (uint64_t)sd.num_rows || (uint64_t)c.rel[k] >= (uint64_t)c.num_relations)) *c.id_bad = 1;
+}
+
 // ---- helper role: waves 8..15 ----
 // The helpers' global loads are all issued from straight-line code at addresses
 // that are valid whatever the slot is (clamped), and what does not apply is
@@ -54,6 +60,7 @@ __device__ __forceinline__ void fused_load_ids(const StepCtx& c, const FusedGeom
   int64_t id = *src;
   if (!is_pos && !sd.uidx)  // the fused route's tables have fewer than 2^31 rows: the draw's 32-bit form (sampled_row)
     id = (int64_t)(((philox_u64(sd.useed, (uint64_t)flat, (uint32_t)s) & 0xffffffffull) * (uint64_t)sd.num_rows) >> 32);
+  fused_check_id(c, sd, k, id);
   id = clamp_index(id, sd.num_rows);
   const int64_t pair = (int64_t)k * c.rk + (is_pos ? sd.slot_pos + q : sd.slot_uni + cc * g.U + u);
   if (real) {
@@ -626,6 +633,7 @@ __global__ __launch_bounds__(kFusedIds) void fused_ids_kernel(StepCtx c) {
   const bool real = j < N && (!is_pos || q < c.B);
   const int64_t flat = (int64_t)kc * U + u;
   int64_t id = is_pos ? sd.idx[(int64_t)k * c.B + min(q, c.B - 1)] : uniform_negative(sd, s, flat);
+  fused_check_id(c, sd, k, id);
   id = clamp_index(id, sd.num_rows);
   if (real) {
     const int64_t pair = (int64_t)k * c.rk + (is_pos ? sd.slot_pos + q : sd.slot_uni + cc * U + u);

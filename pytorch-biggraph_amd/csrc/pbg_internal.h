@@ -79,10 +79,14 @@ struct CosBack {
 struct BatchSums {
   const float* lossrow; const int* violrow; int per_batch; int batches; float* loss_out; unsigned long long* violators;
 };
+// `gate`: asked on the host before the one launch that writes the tables; anything but PBG_OK is returned instead.
+struct UpdateGate {
+  virtual int pass() = 0;
+};
 int row_adagrad_sorted(const uint64_t* keys, const uint32_t* vals, int64_t n, int kbits,
                        float* grad_rows, int dim, float* w0, float* g0, int64_t rows0, float* w1,
                        float* g1, int64_t rows1, float lr, hipStream_t stream, const uint32_t* long_runs = nullptr,
-                       const CosBack* cos_back = nullptr, const BatchSums* sums = nullptr);
+                       const CosBack* cos_back = nullptr, const BatchSums* sums = nullptr, UpdateGate* gate = nullptr);
 
 // ---- plain fp32 batched GEMM on MFMA ----------------------------------------
 // C[b] (M x N, row-major, ldc) = alpha * A[b] * B[b] + beta * C[b], for b in [0, batch).

@@ -932,7 +932,7 @@ __global__ void async_adagrad_dense_kernel(float* __restrict__ p, float* __restr
 template <bool VEC, bool COSB>
 int launch_sorted(int nvec, const uint64_t* keys, const uint32_t* vals, int64_t n, int kbits, float* grad_rows,
                   int dim, float* w0, float* g0, int64_t rows0, float* w1, float* g1, int64_t rows1, float lr,
-                  const uint32_t* long_runs, CosBack cb, BatchSums sums, hipStream_t stream) {
+                  const uint32_t* long_runs, CosBack cb, BatchSums sums, UpdateGate* gate, hipStream_t stream) {
   const int wpb = kRowThreads / kWave;
   const dim3 block(kRowThreads);
   const unsigned tile_blocks = (unsigned)ceil_div(ceil_div(n, kTile), wpb);
@@ -951,6 +951,10 @@ int launch_sorted(int nvec, const uint64_t* keys, const uint32_t* vals, int64_t 
     if (borders > 0)                                                                                              \
       hipLaunchKernelGGL((run_combine_kernel<NV, VEC>), border_grid, block, 0, stream, keys, vals, n, grad_rows, dim,  \
                          leave_mode, long_runs);                                                                   \
+    if (gate) {                                                                                                    \
+      const int allowed = gate->pass();                                                                            \
+      if (allowed != PBG_OK) return allowed;                                                                       \
+    }                                                                                                              \
     if (walk) {                                                                                                    \
       constexpr int R = NV <= 2 ? 8 : (NV <= 4 ? 4 : 2);                                                           \
       hipLaunchKernelGGL((row_walk_kernel<NV, VEC, R, COSB>), walk_grid, block, 0, stream, keys, vals, n, kbits,      \
@@ -985,7 +989,8 @@ int launch_sorted(int nvec, const uint64_t* keys, const uint32_t* vals, int64_t 
 
 int row_adagrad_sorted(const uint64_t* keys, const uint32_t* vals, int64_t n, int kbits, float* grad_rows,
                        int dim, float* w0, float* g0, int64_t rows0, float* w1, float* g1, int64_t rows1, float lr,
-                       hipStream_t stream, const uint32_t* long_runs, const CosBack* cos_back, const BatchSums* sums_in) {
+                       hipStream_t stream, const uint32_t* long_runs, const CosBack* cos_back, const BatchSums* sums_in,
+                       UpdateGate* gate) {
   const BatchSums sums = sums_in ? *sums_in : BatchSums{nullptr, nullptr, 0, 0, nullptr, nullptr};
   if (n <= 0) {  // no gradient rows: a launch that only carries the sums, if any
     if (sums.batches > 0) {
@@ -1000,13 +1005,13 @@ int row_adagrad_sorted(const uint64_t* keys, const uint32_t* vals, int64_t n, in
   if (cos_back) {
     if (dim % 4 != 0) return fail(PBG_ERR_UNSUPPORTED, "row_adagrad: the normalisation backward needs dim %% 4 == 0");
     rc = launch_sorted<true, true>((int)ceil_div(dim / 4, kWave), keys, vals, n, kbits, grad_rows, dim, w0, g0, rows0, w1,
-                                   g1, rows1, lr, long_runs, *cos_back, sums, stream);
+                                   g1, rows1, lr, long_runs, *cos_back, sums, gate, stream);
   } else if (dim % 4 == 0) {
     rc = launch_sorted<true, false>((int)ceil_div(dim / 4, kWave), keys, vals, n, kbits, grad_rows, dim, w0, g0, rows0, w1,
-                                    g1, rows1, lr, long_runs, none, sums, stream);
+                                    g1, rows1, lr, long_runs, none, sums, gate, stream);
   } else {
     rc = launch_sorted<false, false>((int)ceil_div(dim, kWave), keys, vals, n, kbits, grad_rows, dim, w0, g0, rows0, w1, g1,
-                                     rows1, lr, long_runs, none, sums, stream);
+                                     rows1, lr, long_runs, none, sums, gate, stream);
   }
   if (rc != PBG_OK) return rc;
   return check_launch("row_adagrad_sorted");

@@ -2471,7 +2471,90 @@ void launch_reg(const StepCtx& c, hipStream_t s) {
   hipLaunchKernelGGL(reg_reduce_kernel, dim3((unsigned)c.K), dim3(256), 0, s, c);
 }
 
-int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_t s, hipEvent_t* ev) {
+// The arrays of ids a call reads, and the sizes of what they index.
+struct IdArrays {
+  const int64_t* ids[5];
+  int64_t n[5], limit[5];
+  int arrays;
+  int64_t longest;
+};
+IdArrays id_arrays(const pbg_step_desc* d, const pbg_step_buffers* b, const StepCtx& c) {
+  IdArrays a{};
+  const int64_t edges = (int64_t)c.K * c.B;
+  const int64_t rows_r = d->shared_table ? d->num_lhs_rows : d->num_rhs_rows;
+  auto add = [&](const int64_t* ids, int64_t n, int64_t limit) {
+    if (!ids || n <= 0) return;
+    a.ids[a.arrays] = ids;
+    a.n[a.arrays] = n;
+    a.limit[a.arrays++] = limit;
+    if (n > a.longest) a.longest = n;
+  };
+  add(b->lhs, edges, d->num_lhs_rows);
+  add(b->rhs, edges, rows_r);
+  add(b->rel, d->dynamic ? edges : c.K, d->num_relations);
+  if (!b->sample_uniform && !d->all_negs && d->num_uniform_negs > 0) {
+    const int64_t drawn = (int64_t)c.K * c.C * d->num_uniform_negs;
+    if (!d->disable_lhs_negs) add(b->uniform_lhs, drawn, d->num_lhs_rows);
+    if (!d->disable_rhs_negs) add(b->uniform_rhs, drawn, rows_r);
+  }
+  return a;
+}
+// What one thread of `total` (number `t`) sees of an array: is an id outside what it indexes?
+__device__ __forceinline__ bool ids_outside(const IdArrays& a, int which, int64_t t, int64_t total) {
+  const int64_t* __restrict__ ids = a.ids[which];
+  const int64_t n = a.n[which];
+  const uint64_t limit = (uint64_t)a.limit[which];
+  bool out = false;
+  for (int64_t i = t; i < n; i += total) out |= (uint64_t)ids[i] >= limit;
+  return out;
+}
+// Reads a few tens of kilobytes: bound by its launch.
+__global__ __launch_bounds__(256) void check_ids_kernel(IdArrays a, int* __restrict__ bad) {
+  if (ids_outside(a, (int)blockIdx.y, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x))
+    *bad = 1;  // (every writer writes the same)
+}
+
+// A call that is to find ids outside their tables before it changes anything.  The kernel that looks at the ids first
+// (the fused route's own; a kernel of its own on the other routes) leaves its finding in one word of pinned host
+// memory.  The step goes on queuing the kernels that write its workspace only -- they clamp the ids -- and reads that
+// word on the host where the first kernel that writes a table or a parameter comes up: the host waits while the
+// device works.  (A reduction per array and one synchronisation in front of the step cost a call of one batch more
+// than its chunk kernel takes.)
+class IdGate final : public UpdateGate {
+ public:
+  explicit IdGate(int* bad) : bad_(bad) { *bad_ = 0; }
+  ~IdGate() {
+    if (ev_) (void)hipEventDestroy(ev_);
+  }
+  int* word() const { return bad_; }
+  int queue(const IdArrays& a, hipStream_t s) {
+    int64_t blocks = ceil_div(a.longest, 4 * 256);
+    if (blocks > 64) blocks = 64;
+    hipLaunchKernelGGL(check_ids_kernel, dim3((unsigned)blocks, (unsigned)a.arrays), dim3(256), 0, s, a, bad_);
+    return queued(s);
+  }
+  // The kernels that write the word are on the stream.
+  int queued(hipStream_t s) {
+    if (hipEventCreateWithFlags(&ev_, hipEventDisableTiming) != hipSuccess || hipEventRecord(ev_, s) != hipSuccess)
+      return fail(PBG_ERR_LAUNCH, "step: cannot record the id check");
+    return PBG_OK;
+  }
+  // Waits for them (once) and tells what they found.
+  int pass() override {
+    if (!passed_) {
+      if (!ev_ || hipEventSynchronize(ev_) != hipSuccess) return fail(PBG_ERR_LAUNCH, "step: cannot wait for the id check");
+      passed_ = true;
+    }
+    return *bad_ ? fail(PBG_ERR_INDEX, "an id is outside its table") : PBG_OK;
+  }
+
+ private:
+  int* bad_;
+  hipEvent_t ev_ = nullptr;
+  bool passed_ = false;
+};
+
+int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_t s, hipEvent_t* ev, IdGate* gate = nullptr) {
   int rc = validate(desc, true);
   if (rc != PBG_OK) return rc;
   Plan plan;
@@ -2509,6 +2592,11 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
   } join_guard{s};
   hipEvent_t params_done = nullptr;  // set: the operator parameters' kernels were queued on the side stream
   mark(0);
+  const bool gate_in_chunks = gate && plan.fused && plan.max_norm <= 0.f;
+  if (gate && !gate_in_chunks) {
+    if ((rc = gate->queue(id_arrays(desc, bufs, c), s)) != PBG_OK) return rc;
+    if (plan.max_norm > 0.f && (rc = gate->pass()) != PBG_OK) return rc;
+  }
   if ((rc = run_renorm(plan, bufs, s)) != PBG_OK) return rc;
   CosBack cos_back{nullptr, nullptr, nullptr, nullptr};
   const CosBack* cos_back_p = nullptr;
@@ -2579,15 +2667,18 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
       }
     }
     unsigned slot = 0;
+    if (gate_in_chunks) plan.c.id_bad = gate->word();
     if (ss || plan.fl.sliced) {
       plan.c.fused_rowid = plan.fused_rowid;
       if ((rc = fused_ids(c, s)) != PBG_OK) return rc;
+      if (gate_in_chunks && (rc = gate->queued(s)) != PBG_OK) return rc;
     }
     if (ss) {
       slot = ss->next.fetch_add(1) & 7u;
       if (hipEventRecord(ss->fork[slot], s) != hipSuccess) return fail(PBG_ERR_LAUNCH, "step: cannot fork the side stream");
     }
     if ((rc = fused_chunks(c, plan.fl, blocks, s)) != PBG_OK) return rc;  // (queued first: it is to find the machine empty)
+    if (gate_in_chunks && !c.fused_rowid && (rc = gate->queued(s)) != PBG_OK) return rc;
     if (ss) {
       if (hipStreamWaitEvent(ss->stream, ss->fork[slot], 0) != hipSuccess)
         return fail(PBG_ERR_LAUNCH, "step: cannot fork the side stream");
@@ -2602,6 +2693,7 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
       // Two short launches with a handful of waves each: behind the sort on the side stream they run beside the
       // update instead of in front of it.
       if (c.op == PBG_OP_TRANSLATION && !bufs->lhs_global && getenv("PBG_DISABLE_SIDE_PARAMS") == nullptr) {
+        if (gate && (rc = gate->pass()) != PBG_OK) return rc;
         if (hipEventRecord(ss->mid[slot], s) != hipSuccess || hipStreamWaitEvent(ss->stream, ss->mid[slot], 0) != hipSuccess)
           return fail(PBG_ERR_LAUNCH, "step: cannot order the side stream behind the chunk kernel");
         const int params_rc = run_params(desc, bufs, plan, ss->stream, &rel_order, false);
@@ -2650,7 +2742,9 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
     launch_reg(c, s);
     mark(7);
   }
+  if (gate && !params_done && c.op != PBG_OP_NONE && (rc = gate->pass()) != PBG_OK) return rc;
   if (!params_done && (rc = run_params(desc, bufs, plan, s, &rel_order, stream)) != PBG_OK) return rc;
+  if (gate && bufs->lhs_global && (rc = gate->pass()) != PBG_OK) return rc;
   if (bufs->lhs_global) {  // the raw-row gradients are complete and still one per gathered row
     hipLaunchKernelGGL(global_grad_kernel, dim3((unsigned)c.K, (unsigned)(2 * plan.gslices)), dim3(kGlobalHalves * 32), 0,
                        s, c, plan.gth, plan.gslices, plan.fused ? 1 : 0);
@@ -2674,11 +2768,11 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
   const BatchSums sums{c.lossrow, c.violrow, c.C * c.P, c.K, c.loss_out, c.violators};
   if (desc->shared_table) {
     rc = row_adagrad_sorted(skeys, svals, npairs, c.kbits, c.gr, c.D, bufs->w_lhs, bufs->g_lhs,
-                            desc->num_lhs_rows, nullptr, nullptr, 0, desc->lr, s, long_runs, cos_back_p, &sums);
+                            desc->num_lhs_rows, nullptr, nullptr, 0, desc->lr, s, long_runs, cos_back_p, &sums, gate);
   } else {
     rc = row_adagrad_sorted(skeys, svals, npairs, c.kbits, c.gr, c.D, bufs->w_lhs, bufs->g_lhs,
                             desc->num_lhs_rows, bufs->w_rhs, bufs->g_rhs, desc->num_rhs_rows, desc->lr, s, long_runs,
-                            cos_back_p, &sums);
+                            cos_back_p, &sums, gate);
   }
   if (params_done) {
     join_guard.ev2 = nullptr;
@@ -2691,6 +2785,12 @@ int run_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, hipStream_
 
 extern "C" int pbg_train_step(const pbg_step_desc* desc, const pbg_step_buffers* bufs, pbg_stream_t stream) {
   return run_step(desc, bufs, (hipStream_t)stream, nullptr);
+}
+
+extern "C" int pbg_train_step_checked(const pbg_step_desc* desc, const pbg_step_buffers* bufs, int32_t* bad, pbg_stream_t stream) {
+  if (!bad) return fail(PBG_ERR_INVALID, "pbg_train_step_checked: null result word");
+  IdGate gate(bad);
+  return run_step(desc, bufs, (hipStream_t)stream, nullptr, &gate);
 }
 
 extern "C" int pbg_train_step_num_stages(void) { return kStages; }
@@ -2754,6 +2854,78 @@ extern "C" int pbg_model_ranks(const pbg_step_desc* desc, const pbg_step_buffers
                        auc_samples, auc_seed, (unsigned long long*)auc_hits);
   }
   return check_launch("pbg_model_ranks");
+}
+
+namespace {
+// The sums a ranking evaluation reports, in two launches whose partial sums are added in a fixed order.  Reads 20
+// bytes per edge: bound by its launches (ten torch reductions, each read back by itself, took 300 microseconds for
+// the 10000 edges whose ranks take 400).
+constexpr int kRankSums = 14, kRankSumBlocks = 64;
+__device__ __forceinline__ double block_sum(double v, double* sh) {  // 256 threads
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+__global__ __launch_bounds__(256) void rank_sums_kernel(IdArrays a, int64_t count, const int64_t* __restrict__ lhs_rank,
+                                                        const int64_t* __restrict__ rhs_rank,
+                                                        const float* __restrict__ loss_edge, double* __restrict__ partial) {
+  __shared__ double sh[4];
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, total = (int64_t)gridDim.x * 256;
+  double v[kRankSums] = {};
+  for (int64_t i = t; i < count; i += total) {
+    v[0] += (double)loss_edge[i];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int64_t r = (s == 0 ? lhs_rank : rhs_rank)[i];
+      v[1 + 6 * s] += (double)r;
+      v[2 + 6 * s] += r > 0 ? (double)(1.0f / (float)r) : 0.0;
+      v[3 + 6 * s] += r <= 1;
+      v[4 + 6 * s] += r <= 10;
+      v[5 + 6 * s] += r <= 50;
+    }
+  }
+  for (int which = 0; which < a.arrays; ++which)
+    if (ids_outside(a, which, t, total)) v[13] = 1.0;
+#pragma unroll
+  for (int j = 0; j < kRankSums; ++j) {
+    const double sum = block_sum(v[j], sh);
+    if (threadIdx.x == 0) partial[(int64_t)blockIdx.x * kRankSums + j] = sum;
+  }
+}
+__global__ __launch_bounds__(64) void rank_sums_out_kernel(const double* __restrict__ partial, int blocks,
+                                                           const int64_t* __restrict__ auc_hits, double* __restrict__ out) {
+  const int j = threadIdx.x;
+  if (j >= kRankSums) return;
+  double sum = 0.0;
+  for (int b = 0; b < blocks; ++b) sum += partial[(int64_t)b * kRankSums + j];
+  if (j == 6) sum = auc_hits ? (double)auc_hits[0] : 0.0;
+  if (j == 12) sum = auc_hits ? (double)auc_hits[1] : 0.0;
+  out[j] = sum;
+}
+}  // namespace
+
+extern "C" size_t pbg_rank_sums_scratch_bytes(void) { return sizeof(double) * kRankSums * kRankSumBlocks; }
+
+extern "C" int pbg_rank_sums(const pbg_step_desc* desc, const pbg_step_buffers* bufs, int64_t count, const int64_t* lhs_rank,
+                             const int64_t* rhs_rank, const float* loss_edge, const int64_t* auc_hits, double* out,
+                             void* scratch, pbg_stream_t stream) {
+  int rc = validate(desc, false);
+  if (rc != PBG_OK) return rc;
+  Plan plan;
+  make_plan(desc, bufs, &plan);
+  if ((rc = check_buffers(desc, bufs, plan, false)) != PBG_OK) return rc;
+  if (count < 1 || count > (int64_t)plan.c.K * plan.c.B || !lhs_rank || !rhs_rank || !loss_edge || !out || !scratch)
+    return fail(PBG_ERR_INVALID, "pbg_rank_sums: null or empty argument");
+  const IdArrays a = id_arrays(desc, bufs, plan.c);
+  int64_t blocks = ceil_div(count, 256);
+  if (blocks > kRankSumBlocks) blocks = kRankSumBlocks;
+  hipLaunchKernelGGL(rank_sums_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, count, lhs_rank, rhs_rank,
+                     loss_edge, (double*)scratch);
+  hipLaunchKernelGGL(rank_sums_out_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, (const double*)scratch, (int)blocks,
+                     auc_hits, out);
+  return check_launch("pbg_rank_sums");
 }
 
 extern "C" int pbg_model_forward(const pbg_step_desc* desc, const pbg_step_buffers* bufs, float* lhs_pos,

@@ -72,6 +72,7 @@ struct StepCtx {
   float reg_coef;  // N3 regularizer weight (0: none)
   float* regrow;   // [K, 2, B] sum of cubed moduli of each positive's prepared row(s), per side
   float* reg_out;  // [K] or null
+  int* id_bad;     // null, or where the fused route leaves a 1 if an id is outside its table (pinned host memory)
   int* fused_rowid;  // fused route: [K*C, 256] row id of every operand-row slot of a chunk (-1: none), see fused_ids_kernel
 };
 

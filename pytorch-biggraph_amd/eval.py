@@ -4,6 +4,7 @@ MultiRelationEmbedder.forward, i.e. from pbg_model_forward on the GPU; the
 metrics are a handful of reductions over [B] and [B, N] tensors."""
 from statistics import mean
 
+import numpy as np
 import torch
 
 from .batching import AbstractBatchProcessor
@@ -27,6 +28,11 @@ def compute_randomized_auc(pos_: torch.Tensor, neg_: torch.Tensor, num_samples: 
     return float(diff.float().mean())
 
 
+def _sum_of_reciprocals(rank: torch.Tensor) -> float:
+    """The float32 reciprocals, added in float64 and rounded once: the same sum in whatever order it is formed."""
+    return rank.float().reciprocal().double().sum().float().item()
+
+
 def ranking_stats(sides, loss: float, count: int) -> Stats:
     """The sums RankingEvaluator reports for `count` edges (eval.py:57-81).
     sides: (pos [n], neg [n, N]) per side; a side without negatives is skipped.
@@ -39,7 +45,7 @@ def ranking_stats(sides, loss: float, count: int) -> Stats:
     return Stats(
         loss=float(loss),
         pos_rank=average_of_sums(*ranks),
-        mrr=average_of_sums(*(rank.float().reciprocal() for rank in ranks)),
+        mrr=mean(_sum_of_reciprocals(rank) for rank in ranks),
         r1=average_of_sums(*(rank.le(1) for rank in ranks)),
         r10=average_of_sums(*(rank.le(10) for rank in ranks)),
         r50=average_of_sums(*(rank.le(50) for rank in ranks)),
@@ -48,25 +54,12 @@ def ranking_stats(sides, loss: float, count: int) -> Stats:
     )
 
 
-def ranking_stats_from_ranks(ranks, loss: float, count: int, auc_hits=None, auc_samples: int = 0) -> Stats:
-    """The same sums from per-edge ranks (StepRunner.ranks / pbg_model_ranks), one
-    int64 tensor per side that has negatives.  auc_hits[side] of auc_samples random
-    (positive, negative) pairs had positive > negative (util.py:420-428)."""
-    ranks = [r.reshape(-1) for r in ranks]
-    if auc_hits is not None and auc_samples > 0:
-        auc = count * sum(float(h) / auc_samples for h in auc_hits) / len(auc_hits)
-    else:
-        auc = 0.0
-    return Stats(
-        loss=float(loss),
-        pos_rank=average_of_sums(*ranks),
-        mrr=average_of_sums(*(rank.float().reciprocal() for rank in ranks)),
-        r1=average_of_sums(*(rank.le(1) for rank in ranks)),
-        r10=average_of_sums(*(rank.le(10) for rank in ranks)),
-        r50=average_of_sums(*(rank.le(50) for rank in ranks)),
-        auc=auc,
-        count=count,
-    )
+def ranking_stats_from_sums(sides, loss: float, count: int, auc_samples: int) -> Stats:
+    """The same sums from StepRunner.rank_sums: one (ranks, reciprocals, <= 1, <= 10, <= 50, auc hits) per side that
+    has negatives."""
+    sides = [(ranks, float(np.float32(reciprocals)), *rest) for ranks, reciprocals, *rest in sides]
+    pos_rank, mrr, r1, r10, r50, hits = (sum(column) / len(column) for column in zip(*sides))
+    return Stats(loss=loss, pos_rank=pos_rank, mrr=mrr, r1=r1, r10=r10, r50=r50, auc=count * hits / auc_samples, count=count)
 
 
 class RankingEvaluator(AbstractBatchProcessor):
@@ -76,16 +69,14 @@ class RankingEvaluator(AbstractBatchProcessor):
 
     def _process_one_batch(self, model: MultiRelationEmbedder, batch_edges: EdgeList) -> Stats:
         # Without a score filter (the _adjust_scores hook) nothing needs the [B, N] score matrices: ranks,
-        # loss and the AUC count come from one call, per edge.
+        # loss and the AUC count come from one call, summed on the device.
         if type(self)._adjust_scores is RankingEvaluator._adjust_scores and len(batch_edges) > 0:
             count = len(batch_edges)
             kind = batch_edges.get_relation_type_as_scalar() if batch_edges.has_scalar_relation_type() else 0
-            out = model.forward_ranks(batch_edges, loss=self.loss_fn.loss_name, margin=self.loss_fn.fused_margin,
-                                      relation_weight=float(self.relation_weights[kind]), auc_samples=count,
-                                      auc_seed=int(torch.randint(0, 2**62, (1,))))
-            sides = [s for s in range(2) if out.has_negs[s]]
-            return ranking_stats_from_ranks([out.ranks[s] for s in sides], float(out.loss_edge.sum()), count,
-                                            [out.auc_hits[s] for s in sides], count)
+            loss, sides = model.rank_sums(batch_edges, loss=self.loss_fn.loss_name, margin=self.loss_fn.fused_margin,
+                                          relation_weight=float(self.relation_weights[kind]), auc_samples=count,
+                                          auc_seed=int(torch.randint(0, 2**62, (1,))))
+            return ranking_stats_from_sums(sides, loss, count, count)
         with torch.no_grad():
             scores, _ = model(batch_edges)
         self._adjust_scores(scores, batch_edges)

@@ -441,6 +441,21 @@ class MultiRelationEmbedder(nn.Module):
         of every positive among its negatives on either side, the loss -- computed per
         edge on the device without the [B, N] score matrices (pbg_model_ranks;
         reference: eval.py:43-81 over model.py:624-762).  The batch must not be empty."""
+        runner, args, has = self._rank_call(edges, uniform_negs, loss, margin, relation_weight)
+        runner._check_ids(*args[:5])
+        lp, rp, lr, rr, le, hits = runner.ranks(*args, auc_samples, auc_seed)
+        return RankOutput(lp[0], rp[0], (lr[0], rr[0]), le[0], hits, has)
+
+    def rank_sums(self, edges: EdgeList, uniform_negs=None, *, loss: str = "ranking", margin: float = 0.1,
+                  relation_weight: float = 1.0, auc_samples: int = 0, auc_seed: int = 0):
+        """forward_ranks() summed over the batch, on the host: (loss, one StepRunner.rank_sums array per side that has
+        negatives)."""
+        runner, args, has = self._rank_call(edges, uniform_negs, loss, margin, relation_weight)
+        total, sides = runner.rank_sums(*args, auc_samples, auc_seed)
+        return total, [side for side, present in zip(sides, has) if present]
+
+    def _rank_call(self, edges: EdgeList, uniform_negs, loss: str, margin: float, relation_weight: float):
+        """The runner of a batch to rank, the arguments of its call and which sides have negatives."""
         num_pos = len(edges)
         relation_idx, lhs_module, rhs_module = self.resolve(edges)
         if self.num_batch_negs == 0 and self.num_uniform_negs == 0 and not self.relations[relation_idx].all_negs:
@@ -449,17 +464,19 @@ class MultiRelationEmbedder(nn.Module):
             raise ValueError("forward_ranks needs at least one edge")
         w_l, w_r = lhs_module.weight, rhs_module.weight
         dev = w_l.device
-        spec = self.step_spec(relation_idx, num_pos, w_l.shape[1], loss=loss, margin=float(margin))
-        key = ("ranks", relation_idx, num_pos, w_l.data_ptr(), w_r.data_ptr(), loss, float(margin))
+        key = ("ranks", relation_idx, num_pos, w_l.data_ptr(), w_r.data_ptr(), loss, float(margin), self.num_batch_negs,
+               self.num_uniform_negs, float(relation_weight))
         runner = self._runners.get(key)
         if runner is None:
+            spec = self.step_spec(relation_idx, num_pos, w_l.shape[1], loss=loss, margin=float(margin))
             rhs_op, lhs_op = self.operator_tensors(relation_idx)
             glob = self.global_vectors(relation_idx)
+            weights = torch.full((spec.num_relations,), float(relation_weight), dtype=torch.float32, device=dev)
             runner = native.StepRunner(spec, w_l.data, torch.empty(0, device=dev), w_r.data, torch.empty(0, device=dev),
-                                       rhs_op, None, lhs_op, None,
+                                       rhs_op, None, lhs_op, None, relation_weights=weights,
                                        global_embs=None if glob is None else (glob[0].data, glob[1].data))
             self._runners[key] = runner
-        runner.relation_weights.fill_(float(relation_weight))
+        spec = runner.spec
         if uniform_negs is None:
             uniform_negs = self.sample_uniform(lhs_module, rhs_module, spec.num_chunks)
         ul, ur = uniform_negs
@@ -468,13 +485,11 @@ class MultiRelationEmbedder(nn.Module):
         if self.num_dynamic_rels > 0:
             rel = edges.get_relation_type_as_vector().to(dev).contiguous()
         else:
-            rel = torch.zeros(1, dtype=torch.int64, device=dev)  # the runner holds this relation's operator only
+            rel = runner.zero_relation()  # the runner holds this relation's operator only
         weight = edges.weight.to(dev).float().contiguous() if edges.has_weight() else None
-        runner._check_ids(lhs, rhs, rel, ul, ur)
-        lp, rp, lr, rr, le, hits = runner.ranks(lhs, rhs, rel, ul.contiguous() if ul is not None else None,
-                                                ur.contiguous() if ur is not None else None, weight, auc_samples, auc_seed)
         has = (spec.num_negs(self.disable_lhs_negs, w_l.shape[0]) > 0, spec.num_negs(self.disable_rhs_negs, w_r.shape[0]) > 0)
-        return RankOutput(lp[0], rp[0], (lr[0], rr[0]), le[0], hits, has)
+        return runner, (lhs, rhs, rel, ul.contiguous() if ul is not None else None,
+                        ur.contiguous() if ur is not None else None, weight), has
 
     def forward(self, edges: EdgeList, uniform_negs=None) -> Tuple[Scores, Optional[FloatTensorType]]:
         """Scores of a batch and the regularizer's value, None without a
@@ -511,7 +526,7 @@ class MultiRelationEmbedder(nn.Module):
         if self.num_dynamic_rels > 0:
             rel = edges.get_relation_type_as_vector().to(dev).contiguous()
         else:
-            rel = torch.zeros(1, dtype=torch.int64, device=dev)  # the runner holds this relation's operator only
+            rel = runner.zero_relation()  # the runner holds this relation's operator only
         runner._check_ids(lhs, rhs, rel, ul, ur)  # IndexError, as F.embedding raises it (model.py:60-61)
         lp, rp, ln, rn = runner.forward(lhs, rhs, rel, ul.contiguous() if ul is not None else None,
                                         ur.contiguous() if ur is not None else None)

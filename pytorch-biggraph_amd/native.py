@@ -7,6 +7,7 @@ import ctypes
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -256,6 +257,28 @@ class StepSpec:
         return (self.chunk_size if self.num_batch_negs > 0 else 0) + self.num_uniform_negs
 
 
+class _HostResults:
+    """Pinned host memory that the kernels write a call's results to, so that the host reads them after one
+    synchronisation instead of copying each tensor back by itself."""
+
+    def __init__(self, k: int) -> None:
+        sums = 14  # pbg_rank_sums
+        self._raw = torch.zeros(8 * (1 + sums + 2 * k) + 8 * k, dtype=torch.uint8, pin_memory=True)
+        raw, base = self._raw.numpy(), self._raw.data_ptr()
+        at = [0]
+
+        def take(count, dtype):
+            first = at[0]
+            at[0] += count * dtype().itemsize
+            return raw[first:at[0]].view(dtype), base + first
+
+        self.bad, self.bad_ptr = take(2, np.int32)
+        self.sums, self.sums_ptr = take(sums, np.float64)
+        self.violators, self.violators_ptr = take(2 * k, np.int64)
+        self.loss, self.loss_ptr = take(k, np.float32)
+        self.reg, self.reg_ptr = take(k, np.float32)
+
+
 class StepRunner:
     """Owns the descriptor, the workspace and the output buffers of
     pbg_train_step / pbg_model_forward for one configuration and one pair of
@@ -330,6 +353,8 @@ class StepRunner:
         self.loss_out = torch.zeros(k, dtype=torch.float32, device=dev)
         self.violators_out = torch.zeros((k, 2), dtype=torch.int64, device=dev)
         self.reg_out = torch.zeros(k, dtype=torch.float32, device=dev)  # Stats.reg of each batch
+        self._host: Optional[_HostResults] = None
+        self._zero_rel: Optional[torch.Tensor] = None
 
     @staticmethod
     def _op_pair(params: Dict[str, torch.Tensor]) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor]]:
@@ -404,11 +429,9 @@ class StepRunner:
         from `uniform_seed` (sample_uniform_negatives shows which).
 
         The kernels clamp an id outside its table instead of failing.  With
-        `check_ids` the ids are range-checked first (one reduction per array and
-        one host synchronisation) and an IndexError is raised as F.embedding does
-        in the reference (model.py:60-61)."""
-        if check_ids:
-            self._check_ids(lhs, rhs, rel, uniform_lhs, uniform_rhs)
+        `check_ids` an id out of range raises IndexError, as F.embedding does in the
+        reference (model.py:60-61), before anything is trained
+        (pbg_train_step_checked; the host waits for the check of the ids)."""
         bufs = self._buffers(lhs, rhs, rel, uniform_lhs, uniform_rhs, edge_weight, uniform_seed)
         if stats_out is not None:
             loss, viol = stats_out
@@ -416,7 +439,39 @@ class StepRunner:
             if _need(loss, torch.float32, "stats_out[0]").numel() != k or _need(viol, torch.int64, "stats_out[1]").numel() != 2 * k:
                 raise ValueError(f"stats_out must be (loss[{k}], violators[{k}, 2])")
             bufs.loss_out, bufs.violators_out = _ptr(loss), _ptr(viol)
-        check(_lib.lib().pbg_train_step(ctypes.byref(self.desc), ctypes.byref(bufs), _stream()))
+        self._step(bufs, _stream(), check_ids, lhs, rhs, rel, uniform_lhs, uniform_rhs)
+
+    def train_stats(self, lhs, rhs, rel, uniform_lhs=None, uniform_rhs=None, edge_weight=None, check_ids: bool = False):
+        """train(), and its statistics on the host: (loss [K] float32, reg [K] float32, violators [K, 2] int64) as
+        numpy arrays that the next call overwrites.  The kernels write them to host memory; the call ends with the
+        one synchronisation that takes."""
+        bufs = self._buffers(lhs, rhs, rel, uniform_lhs, uniform_rhs, edge_weight)
+        host = self._host_results()
+        bufs.loss_out, bufs.violators_out, bufs.reg_out = host.loss_ptr, host.violators_ptr, host.reg_ptr
+        stream = torch.cuda.current_stream()
+        self._step(bufs, stream.cuda_stream, check_ids, lhs, rhs, rel, uniform_lhs, uniform_rhs)
+        stream.synchronize()
+        return host.loss, host.reg, host.violators.reshape(-1, 2)
+
+    def _host_results(self) -> _HostResults:
+        if self._host is None:
+            self._host = _HostResults(self.spec.num_workers)
+        return self._host
+
+    def zero_relation(self) -> torch.Tensor:
+        """[K] zeros: the relation argument of a runner that holds one relation's operator only."""
+        if self._zero_rel is None:
+            self._zero_rel = torch.zeros(self.spec.num_workers, dtype=torch.int64, device=self.device)
+        return self._zero_rel
+
+    def _step(self, bufs: StepBuffers, stream: int, check_ids: bool, *ids) -> None:
+        if not check_ids:
+            check(_lib.lib().pbg_train_step(ctypes.byref(self.desc), ctypes.byref(bufs), stream))
+            return
+        status = _lib.lib().pbg_train_step_checked(ctypes.byref(self.desc), ctypes.byref(bufs), self._host_results().bad_ptr, stream)
+        if status == _lib.PBG_ERR_INDEX:
+            self._check_ids(*ids)  # names the array and the id
+        check(status)
 
     def _check_ids(self, lhs, rhs, rel, uniform_lhs, uniform_rhs) -> None:
         bounds = []
@@ -493,6 +548,38 @@ class StepRunner:
                                          _ptr(lhs_rank), _ptr(rhs_rank), _ptr(loss_edge), int(auc_samples),
                                          auc_seed & (2**64 - 1), _ptr(hits), _stream()))
         return lhs_pos, rhs_pos, lhs_rank, rhs_rank, loss_edge, hits
+
+    def rank_sums(self, lhs, rhs, rel, uniform_lhs=None, uniform_rhs=None, edge_weight=None, auc_samples: int = 0,
+                  auc_seed: int = 0, check_ids: bool = True):
+        """ranks() reduced to what an evaluation reports (pbg_rank_sums), on the host: (loss, sides), `sides` one
+        array (sum of ranks, sum of 1 / rank, ranks <= 1, <= 10, <= 50, auc_hits) per side, lhs first.  With `check_ids`
+        an id outside its table raises IndexError."""
+        if check_ids and self.desc.max_norm > 0:  # the lookups change the tables
+            self._check_ids(lhs, rhs, rel, uniform_lhs, uniform_rhs)
+        bufs = self._buffers(lhs, rhs, rel, uniform_lhs, uniform_rhs, edge_weight)
+        k, b = self.spec.num_workers, self.spec.batch_size
+        stream = torch.cuda.current_stream()
+        count, lib, raw_stream = k * b, _lib.lib(), stream.cuda_stream
+        scratch_bytes = lib.pbg_rank_sums_scratch_bytes()
+        raw = torch.empty(count * 28 + 16 + scratch_bytes, dtype=torch.uint8, device=self.device)
+        base = raw.data_ptr()
+        scratch = base
+        hits = base + scratch_bytes if auc_samples > 0 else None
+        lhs_rank = base + scratch_bytes + 16
+        rhs_rank = lhs_rank + 8 * count
+        lhs_pos = rhs_rank + 8 * count
+        rhs_pos = lhs_pos + 4 * count
+        loss_edge = rhs_pos + 4 * count
+        check(lib.pbg_model_ranks(ctypes.byref(self.desc), ctypes.byref(bufs), lhs_pos, rhs_pos, lhs_rank, rhs_rank, loss_edge,
+                                  int(auc_samples), auc_seed & (2**64 - 1), hits, raw_stream))
+        host = self._host_results()
+        check(lib.pbg_rank_sums(ctypes.byref(self.desc), ctypes.byref(bufs), count, lhs_rank, rhs_rank, loss_edge, hits,
+                                host.sums_ptr, scratch, raw_stream))
+        stream.synchronize()
+        out = host.sums.tolist()
+        if check_ids and out[13] != 0:
+            self._check_ids(lhs, rhs, rel, uniform_lhs, uniform_rhs)
+        return out[0], (out[1:7], out[7:13])
 
     def forward(self, lhs, rhs, rel, uniform_lhs=None, uniform_rhs=None):
         """Scores only: (lhs_pos[K,B], rhs_pos[K,B], lhs_neg[K,B,Nl], rhs_neg[K,B,Nr])."""

@@ -110,15 +110,14 @@ class Trainer(AbstractBatchProcessor):
         if model.num_dynamic_rels > 0:
             rel = batch_edges.get_relation_type_as_vector().to(dev).contiguous()
         else:
-            rel = torch.zeros(1, dtype=torch.int64, device=dev)
+            rel = runner.zero_relation()
         weight = batch_edges.weight
         if weight is not None:
             weight = weight.to(device=dev, dtype=torch.float32).expand(num_pos).contiguous()
         # An id outside its table raises IndexError here, as F.embedding does in the reference (model.py:60-61);
-        # the kernels themselves would clamp it.  The check's synchronisation is one this method has anyway.
-        runner.train(lhs, rhs, rel, ul.contiguous() if ul is not None else None,
-                     ur.contiguous() if ur is not None else None, weight, check_ids=self.check_ids)
-        # the reference reads loss and both violator counts on the host for every batch (train_cpu.py:95-101)
-        viol = runner.violators_out[0].tolist()
-        return Stats(loss=float(runner.loss_out[0]), reg=float(runner.reg_out[0]), violators_lhs=int(viol[0]), violators_rhs=int(viol[1]),
+        # the kernels themselves would clamp it.
+        # The reference reads loss and both violator counts on the host for every batch (train_cpu.py:95-101).
+        loss, reg, viol = runner.train_stats(lhs, rhs, rel, ul.contiguous() if ul is not None else None,
+                                             ur.contiguous() if ur is not None else None, weight, check_ids=self.check_ids)
+        return Stats(loss=float(loss[0]), reg=float(reg[0]), violators_lhs=int(viol[0, 0]), violators_rhs=int(viol[0, 1]),
                      count=num_pos)
