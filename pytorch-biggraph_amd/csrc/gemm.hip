@@ -47,56 +47,75 @@ struct Operand {
   float v[kUnits][8];
   const float* base;
   int ld, row[kUnits], rmax;
-  bool vec;  // every vector load of a full step is aligned and in bounds
+  bool vec;  // every vector load is aligned, and whole or absent
 
   static __device__ __forceinline__ int unit_group(int u) {
-    return KMAJOR ? (threadIdx.x >> 6) & 3 : (threadIdx.x + u * THREADS) & 3;
+    // (of a k-major operand: the same for the wave, so that a row's address is a scalar and the lane's offset 32 bits)
+    return KMAJOR ? __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3) : (threadIdx.x + u * THREADS) & 3;
   }
   static __device__ __forceinline__ int unit_row(int u) {
     if (KMAJOR) return (threadIdx.x >> 8) * (64 * kUnits) + (threadIdx.x & 63) * kUnits + u;
     return (threadIdx.x + u * THREADS) >> 2;
   }
 
-  __device__ __forceinline__ void start(const float* base_, int ld_, int r0, int rmax_, int aligned_to) {
+  __device__ __forceinline__ void start(const float* base_, int ld_, int r0, int rmax_, int kmax, int aligned_to) {
     base = base_;
     ld = ld_;
     rmax = rmax_;
-    vec = KMAJOR ? (kUnits == 1 || (aligned_to >= 2 && rmax % 2 == 0)) : aligned_to >= 4;
+    vec = KMAJOR ? (kUnits == 1 || (aligned_to >= 2 && rmax % 2 == 0)) : aligned_to >= 4 && kmax % 4 == 0 && kmax > 0;
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) row[u] = min(r0 + unit_row(u), rmax - 1);
     if (KMAJOR && kUnits == 2 && vec) row[0] = min(r0 + unit_row(0), rmax - 2);
   }
 
-  // Whole vectors of a step that lies inside [0, kmax); of a k-major operand only the first call fetches (all units).
-  __device__ __forceinline__ void fetch_full(int k0, int u) {
+  // Whole vectors of a step; of a k-major operand only the first call fetches (all units).  LAST: the step may reach past
+  // kmax: those vectors are read from inside and zeroed.
+  template <bool LAST>
+  __device__ __forceinline__ void fetch_vec(int k0, int u, int kmax) {
     if constexpr (!KMAJOR) {
-      const float* p = base + (int64_t)row[u] * ld + k0 + 4 * unit_group(u);
-      const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 16);
+      const int k = k0 + 4 * unit_group(u);
+      const float* p = base + (int64_t)row[u] * ld;
+      float4 x = *reinterpret_cast<const float4*>(p + (LAST ? min(k, kmax - 4) : k));
+      float4 y = *reinterpret_cast<const float4*>(p + (LAST ? min(k + 16, kmax - 4) : k + 16));
+      if constexpr (LAST) {
+        if (k >= kmax) x = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (k + 16 >= kmax) y = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
       v[u][0] = x.x; v[u][1] = x.y; v[u][2] = x.z; v[u][3] = x.w;
       v[u][4] = y.x; v[u][5] = y.y; v[u][6] = y.z; v[u][7] = y.w;
     } else if (u == 0) {
-      const float* p = base + (int64_t)(k0 + 4 * unit_group(0)) * ld + row[0];
+      const uint32_t at = 4u * (uint32_t)row[0];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float* q = p + (int64_t)((j & 3) + 16 * (j >> 2)) * ld;
+        const int k = k0 + 4 * unit_group(0) + (j & 3) + 16 * (j >> 2);
+        const char* q = reinterpret_cast<const char*>(base + (int64_t)(LAST ? min(k, kmax - 1) : k) * ld);
         if constexpr (kUnits == 2) {
-          const float2 x = *reinterpret_cast<const float2*>(q);
+          const float2 x = *reinterpret_cast<const float2*>(q + at);
           v[0][j] = x.x;
           v[1][j] = x.y;
         } else {
-          v[0][j] = *q;
+          v[0][j] = *reinterpret_cast<const float*>(q + at);
+        }
+        if constexpr (LAST) {
+#pragma unroll
+          for (int w = 0; w < kUnits; ++w) v[w][j] = k < kmax ? v[w][j] : 0.f;
         }
       }
     }
   }
 
   __device__ __forceinline__ void fetch(int k0, int kmax) {
-    if (vec && k0 + kStepK <= kmax) {
+    if (vec) {
+      if (k0 + kStepK <= kmax) {
 #pragma unroll
-      for (int u = 0; u < kUnits; ++u) fetch_full(k0, u);
+        for (int u = 0; u < kUnits; ++u) fetch_vec<false>(k0, u, kmax);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) fetch_vec<true>(k0, u, kmax);
+      }
       return;
     }
-    // the last step of an operand whose k is no multiple of 32, or unaligned rows: value by value, zero past kmax
+    // unaligned rows, or k no multiple of 4 along them: value by value, zero past kmax
 #pragma unroll
     for (int u = 0; u < kUnits; ++u)
 #pragma unroll
@@ -134,7 +153,8 @@ struct GemmShape {
   static constexpr size_t kLds = 2 * sizeof(uint4) * kStage;
 };
 
-template <int WM, int WN, int TM, int TN, bool A_KMAJOR, bool B_KMAJOR, bool HALF>
+// BFIRST: GemmArgs.b_first
+template <int WM, int WN, int TM, int TN, bool A_KMAJOR, bool B_KMAJOR, bool HALF, bool BFIRST>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int tiles_m, int tiles_n, int a_align, int b_align) {
   using Shape = GemmShape<WM, WN, TM, TN, HALF>;
   constexpr int P = Shape::kParts;
@@ -157,8 +177,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int t
 
   Operand<RA, Shape::kThreads, A_KMAJOR, HALF> oa;
   Operand<RB, Shape::kThreads, B_KMAJOR, HALF> ob;
-  oa.start(g.a + (int64_t)batch * g.stride_a, g.lda, m0, g.m, a_align);
-  ob.start(g.b + (int64_t)batch * g.stride_b + (g.b_index ? g.b_index[batch] * g.b_index_stride : 0), g.ldb, n0, g.n, b_align);
+  oa.start(g.a + (int64_t)batch * g.stride_a, g.lda, m0, g.m, g.k, a_align);
+  ob.start(g.b + (int64_t)batch * g.stride_b + (g.b_index ? g.b_index[batch] * g.b_index_stride : 0), g.ldb, n0, g.n, g.k, b_align);
 
   // Blocked summation: `acc` collects kFoldSteps steps, then is folded into `tot`.  A single accumulator over k = 1000
   // rounds in proportion to the running sum at every step, coherently when the terms are alike (a power-law batch repeats
@@ -214,12 +234,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int t
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, fa[0]), __builtin_bit_cast(half8v, fb[j][0]), acc[i][j], 0, 0, 0);
       } else {
         // part pairs in ascending size; the tiles of a pair follow each other, so that no instruction waits for the last
-        constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+        constexpr int first[6] = {0, 2, 1, 0, 1, 0}, second[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
         for (int q = 0; q < 6; ++q)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[pa[q]]), __builtin_bit_cast(bf16x8, fb[j][pb[q]]), acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa[BFIRST ? second[q] : first[q]]),
+                                                                __builtin_bit_cast(bf16x8, fb[j][BFIRST ? first[q] : second[q]]), acc[i][j], 0, 0, 0);
       }
       if constexpr (decltype(more)::value) {
 #pragma unroll
@@ -228,11 +249,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int t
           if constexpr (decltype(full)::value) {
             // (a k-major operand's loads fill all its units: they go out behind its last one)
             if (u < oa.kUnits) {
-              if (!A_KMAJOR) oa.fetch_full((kt + 2) * kStepK, u);
-              else if (u == oa.kUnits - 1) oa.fetch_full((kt + 2) * kStepK, 0);
+              if (!A_KMAJOR) oa.template fetch_vec<false>((kt + 2) * kStepK, u, g.k);
+              else if (u == oa.kUnits - 1) oa.template fetch_vec<false>((kt + 2) * kStepK, 0, g.k);
             } else {
-              if (!B_KMAJOR) ob.fetch_full((kt + 2) * kStepK, u - oa.kUnits);
-              else if (u == kUnits - 1) ob.fetch_full((kt + 2) * kStepK, 0);
+              if (!B_KMAJOR) ob.template fetch_vec<false>((kt + 2) * kStepK, u - oa.kUnits, g.k);
+              else if (u == kUnits - 1) ob.template fetch_vec<false>((kt + 2) * kStepK, 0, g.k);
             }
           }
         }
@@ -270,6 +291,43 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int t
 
   // D[i = 4 * (lane / 16) + r][j = lane % 16] lives in register r of the lane.
   float* __restrict__ c = g.c + (int64_t)batch * g.stride_c;
+  if constexpr (!HALF) {
+    // The split turns an infinite value (and one that rounds up to an infinite bf16 number) into NaN: a wave that finds one
+    // in its part of the tile sums it again, entry by entry, without the split.
+    float any = 0.f;  // NaN once an infinite or NaN value was added times 0
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) any = fmaf(0.f, tot[i][j][r] + acc[i][j][r], any);
+    if (__any(any != 0.f)) {  // (NaN compares unequal)
+      const int64_t step_a = A_KMAJOR ? g.lda : 1, row_a = A_KMAJOR ? 1 : g.lda;
+      const int64_t step_b = B_KMAJOR ? g.ldb : 1, row_b = B_KMAJOR ? 1 : g.ldb;
+#pragma unroll 1
+      for (int e = 0; e < TM * TN * 4; ++e) {
+        const int row = m0 + wm0 + (e / (4 * TN)) * 16 + 4 * (lane >> 4) + (e & 3);
+        const int col = n0 + wn0 + (e / 4 % TN) * 16 + (lane & 15);
+        if (row < g.m && col < g.n) {
+          float* dst = c + (int64_t)row * g.ldc + col;
+          const float* pa = oa.base + row * row_a;
+          const float* pb = ob.base + col * row_b;
+          float sum = 0.f, part = 0.f;
+#pragma unroll 1
+          for (int k = 0; k < g.k; ++k, pa += step_a, pb += step_b) {
+            part = fmaf(*pa, *pb, part);
+            if ((k + 1) % (kFoldSteps * kStepK) == 0) {
+              sum += part;
+              part = 0.f;
+            }
+          }
+          const float v = g.alpha * (sum + part);
+          *dst = g.beta != 0.f ? v + g.beta * *dst : v;
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -297,11 +355,11 @@ int row_alignment(const float* p, int ld, int64_t stride, int64_t more) {
   return bits % 4 == 0 ? 4 : bits % 2 == 0 ? 2 : 1;
 }
 
-template <int WM, int WN, int TM, int TN, bool AK, bool BK, bool HALF>
+template <int WM, int WN, int TM, int TN, bool AK, bool BK, bool HALF, bool BFIRST = false>
 int launch_one(const GemmArgs& g, hipStream_t stream) {
   using Shape = GemmShape<WM, WN, TM, TN, HALF>;
   static LdsLimit limit;
-  auto kernel = gemm_kernel<WM, WN, TM, TN, AK, BK, HALF>;
+  auto kernel = gemm_kernel<WM, WN, TM, TN, AK, BK, HALF, BFIRST>;
   const int rc = reserve_lds((const void*)kernel, &limit, Shape::kLds);
   if (rc != PBG_OK) return rc;
   const int64_t tm = ceil_div(g.m, Shape::kRowsA), tn = ceil_div(g.n, Shape::kRowsB);
@@ -313,7 +371,9 @@ int launch_one(const GemmArgs& g, hipStream_t stream) {
 
 template <int WM, int WN, int TM, int TN, bool HALF>
 int launch(const GemmArgs& g, hipStream_t stream) {
-  if (!g.a_kmajor && !g.b_kmajor) return launch_one<WM, WN, TM, TN, false, false, HALF>(g, stream);
+  if (!g.a_kmajor && !g.b_kmajor)
+    return g.b_first && !HALF ? launch_one<WM, WN, TM, TN, false, false, HALF, !HALF>(g, stream)
+                              : launch_one<WM, WN, TM, TN, false, false, HALF>(g, stream);
   if (!g.a_kmajor) return launch_one<WM, WN, TM, TN, false, true, HALF>(g, stream);
   if (!g.b_kmajor) return launch_one<WM, WN, TM, TN, true, false, HALF>(g, stream);
   return launch_one<WM, WN, TM, TN, true, true, HALF>(g, stream);

@@ -107,6 +107,9 @@ struct GemmArgs {
   // 1: every value of A and B is a float16 number (held as fp32): the products run on the fp16 matrix
   // instructions, still summed in fp32, and C is rounded to float16 numbers (torch.bmm on Half tensors)
   int half = 0;
+  // 1: the split products' parts are taken in B's order instead of A's.  An entry of A B^T comes out the same, to the last
+  // bit, as the entry of B A^T over the same two rows that is computed without it (both operands k-contiguous; otherwise ignored).
+  int b_first = 0;
 };
 int gemm_f32(const GemmArgs& args, hipStream_t stream);
 

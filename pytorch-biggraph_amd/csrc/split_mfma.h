@@ -14,8 +14,9 @@
 // error 0.8-6.2e-8 (2.7e-7 on constant rows) where the fp32 instruction gives 1.0-7.3e-8 (9.3e-7): an instruction rounds
 // once per 32 values of k here and once per value there.
 //
-// Not covered by the argument: |x| < 2^-110 (l falls below bf16's range; an absolute error below 2^-133) and infinite
-// values, whose product comes out NaN.
+// Not covered by the argument: |x| < 2^-110 (l falls below bf16's range; an absolute error below 2^-133), and infinite
+// values and those within 2^-9 of the largest fp32 number (h is infinite), whose products come out NaN: the caller has to
+// look for NaN and compute those entries otherwise.
 #pragma once
 
 #include "pbg_internal.h"

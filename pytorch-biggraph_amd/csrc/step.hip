@@ -2232,6 +2232,9 @@ int run_scores(const Plan& plan, hipStream_t stream) {
     g.c = sd.s; g.stride_c = (int64_t)P * sd.nn; g.ldc = sd.nn;
     g.m = P; g.n = sd.nn; g.k = D; g.batch = K * C; g.alpha = 1.f; g.beta = 0.f;
     g.half = c.half;
+    // The positive score is side 0's (positive_scores): a negative of side 1 that is the positive's own entity is the same
+    // pair with the operands exchanged, and has to tie with it exactly (a rank counts ties, a hinge stands at its margin).
+    g.b_first = s;
     if ((rc = gemm_f32(g, stream)) != PBG_OK) return rc;
   }
   return check_launch("step forward");
