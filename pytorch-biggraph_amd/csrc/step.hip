@@ -295,8 +295,9 @@ struct ScoreRow {
 
   // score of column j as the model returns it (model.py:234-246,836-839); `live`
   // is false where the value is a constant with no gradient
-  __device__ __forceinline__ float at(int j, bool* live) const {
-    float t = raw[j];
+  __device__ __forceinline__ float at(int j, bool* live) const { return finish(j, raw[j], live); }
+  // the same from the chunk score row's value
+  __device__ __forceinline__ float finish(int j, float t, bool* live) const {
     bool ok = true;
     if (cmp == PBG_CMP_L2) {
       const float qd = fmaf(-2.0f, t, bn[j]) + a2;
@@ -685,28 +686,63 @@ __global__ __launch_bounds__(kRowThreads) void scores_out_kernel(StepCtx c, floa
 // number of negatives scoring at least as high, masked entries (-1e9) included as they are in the
 // reference's matrices -- and the edge's loss.  One wave per edge reads the chunk's score rows where the
 // score GEMMs left them.
+//
+// Bound by reading the scores once (160 MB for 10000 edges against 2 x 2000 candidates).  HELD: a lane keeps its scores of a row
+// of at most 64 * HELD columns (dot or cos scores without biases, which need no further arrays), all loaded at once from clamped addresses (one load at a time, and a second pass for the
+// softmax's sum, took 117 us for those); HELD = 0: rows of any length, read once per pass.
+template <int HELD>
 __device__ __forceinline__ void row_rank_and_loss(int loss, float margin, const ScoreRow& sr, int nn, float pos, int lane,
                                                   float* loss_acc, int* at_least) {
   bool live;
   int ge = 0;
   float mx = pos;
-  for (int j = lane; j < nn; j += kWave) {
-    const float t = sr.at(j, &live);
-    if (t >= pos) ++ge;
+  float t[HELD > 0 ? HELD : 1];
+  if constexpr (HELD > 0) {
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) t[u] = sr.raw[min(lane + u * kWave, nn - 1)];
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) {
+      const int j = lane + u * kWave;
+      if ((j < sr.nb && (j == sr.i || j >= sr.masked_from)) || j == sr.own) t[u] = -1e9f;
+      ge += j < nn && t[u] >= pos;
+      if (j >= nn) t[u] = -INFINITY;  // adds nothing to any loss
+    }
     if (loss == PBG_LOSS_RANKING) {
-      const float x = (t - pos) + margin;
-      if (x > 0.f) *loss_acc += x;
+#pragma unroll
+      for (int u = 0; u < HELD; ++u) *loss_acc += fmaxf((t[u] - pos) + margin, 0.f);
     } else if (loss == PBG_LOSS_LOGISTIC) {
       float sg;
-      *loss_acc += softplus_sigmoid(t, &sg) / (float)nn;
+#pragma unroll
+      for (int u = 0; u < HELD; ++u) *loss_acc += softplus_sigmoid(t[u], &sg) / (float)nn;
     } else {
-      mx = fmaxf(mx, t);
+#pragma unroll
+      for (int u = 0; u < HELD; ++u) mx = fmaxf(mx, t[u]);
+    }
+  } else {
+    for (int j = lane; j < nn; j += kWave) {
+      const float tj = sr.at(j, &live);
+      if (tj >= pos) ++ge;
+      if (loss == PBG_LOSS_RANKING) {
+        const float x = (tj - pos) + margin;
+        if (x > 0.f) *loss_acc += x;
+      } else if (loss == PBG_LOSS_LOGISTIC) {
+        float sg;
+        *loss_acc += softplus_sigmoid(tj, &sg) / (float)nn;
+      } else {
+        mx = fmaxf(mx, tj);
+      }
     }
   }
   if (loss == PBG_LOSS_SOFTMAX) {
     mx = wave_max(mx);
     float z = 0.f;
-    for (int j = lane; j < nn; j += kWave) z += exp_below(sr.at(j, &live), mx);
+    if constexpr (HELD > 0) {
+#pragma unroll
+      for (int u = 0; u < HELD; ++u)
+        z += exp_below(t[u], mx);
+    } else {
+      for (int j = lane; j < nn; j += kWave) z += exp_below(sr.at(j, &live), mx);
+    }
     z = wave_sum(z) + exp_below(pos, mx);
     if (lane == 0) *loss_acc += (mx + logf(z)) - pos;
   } else if (loss == PBG_LOSS_LOGISTIC) {
@@ -715,6 +751,7 @@ __device__ __forceinline__ void row_rank_and_loss(int loss, float margin, const 
   *at_least = wave_sum_int(ge);
 }
 
+template <int HELD>
 __global__ __launch_bounds__(kRowThreads) void ranks_out_kernel(StepCtx c, float* __restrict__ lhs_pos,
                                                                 float* __restrict__ rhs_pos,
                                                                 int64_t* __restrict__ lhs_rank,
@@ -740,7 +777,7 @@ __global__ __launch_bounds__(kRowThreads) void ranks_out_kernel(StepCtx c, float
     }
     ScoreRow sr = score_row(c, s, kc, cc, i);
     int ge;
-    row_rank_and_loss(c.loss, c.margin, sr, nn, posv[s], lane, &loss_acc, &ge);
+    row_rank_and_loss<HELD>(c.loss, c.margin, sr, nn, posv[s], lane, &loss_acc, &ge);
     rank[s] = (int64_t)ge + 1;
   }
   const float loss_row = wave_sum(loss_acc) * w;
@@ -2848,7 +2885,12 @@ extern "C" int pbg_model_ranks(const pbg_step_desc* desc, const pbg_step_buffers
   if ((rc = run_prep(plan, s)) != PBG_OK) return rc;
   if ((rc = run_operator_forward(plan, s, &rel_order)) != PBG_OK) return rc;
   if ((rc = run_scores(plan, s)) != PBG_OK) return rc;
-  hipLaunchKernelGGL(ranks_out_kernel, wave_grid((int64_t)c.K * c.B), dim3(kRowThreads), 0, s, c, lhs_pos, rhs_pos, lhs_rank,
+  const int longest = std::max(c.side[0].nn, c.side[1].nn);
+  const auto ranks_out = is_distance(c.cmp) || c.bias || longest > 32 * kWave ? ranks_out_kernel<0>
+                         : longest <= 4 * kWave                             ? ranks_out_kernel<4>
+                         : longest <= 16 * kWave                            ? ranks_out_kernel<16>
+                                                                            : ranks_out_kernel<32>;
+  hipLaunchKernelGGL(ranks_out, wave_grid((int64_t)c.K * c.B), dim3(kRowThreads), 0, s, c, lhs_pos, rhs_pos, lhs_rank,
                      rhs_rank, loss_edge);
   if (auc_samples > 0) {
     static_assert(sizeof(unsigned long long) == sizeof(int64_t), "auc_hits is written as two 64-bit counters");
