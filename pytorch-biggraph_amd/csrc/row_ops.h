@@ -325,11 +325,19 @@ __device__ __forceinline__ float sigmoidf(float z) {
 // included) goes through it, so that terms that must cancel still do.
 __device__ __forceinline__ float exp_below(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * 1.4426950408889634f); }
 
-// softplus(z) and sigmoid(z) from one exponential (the same values as the two functions above)
+// softplus(z) and sigmoid(z) from one exponential e = e^-|z|, with the hardware's log2 and reciprocal (1 ulp each) made good
+// where they alone would lose digits: u = fl(1 + e) is off by c = e - (u - 1) exactly, so log(1 + e) = log(u) + c / u to first
+// order, and the reciprocal of u + c is one Newton step away from that of u.  log1pf and a division took three quarters of the
+// kernel's instructions and made the logistic loss arithmetic-bound (51 M scores staged: 361 us).  Against float64,
+// z in [-5, 5]: the sigmoid is off by 3.2e-8 rms, 1.5e-7 at most (4.2e-8 and 1.7e-7 with the division); 361 -> 240 us.
 __device__ __forceinline__ float softplus_sigmoid(float z, float* sigmoid) {
   const float e = expf(-fabsf(z));
-  *sigmoid = (z >= 0.f ? 1.0f : e) / (1.0f + e);
-  return fmaxf(z, 0.f) + log1pf(e);
+  const float u = 1.0f + e, c = e - (u - 1.0f);
+  const float r0 = __builtin_amdgcn_rcpf(u);
+  const float r = fmaf(fmaf(-c, r0, fmaf(-u, r0, 1.0f)), r0, r0);
+  *sigmoid = (z >= 0.f ? 1.0f : e) * r;
+  const float l = __builtin_amdgcn_logf(u);
+  return fmaxf(z, 0.f) + fmaf(l, 0.693147182f, fmaf(l, -1.90465421e-9f, c * r));  // ln 2 = 0.693147182 - 1.90465421e-9
 }
 
 }  // namespace pbg
