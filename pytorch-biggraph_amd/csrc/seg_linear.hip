@@ -406,33 +406,62 @@ __global__ __launch_bounds__(kThreads, 4) void seg_linear_update_kernel(
     }
   };
 
+  // One Adagrad step per run and matrix cell is most of this kernel's arithmetic when the runs are short (22 000 runs of two
+  // or three edges each at 128 000 edges over 500 skewed relations: 1.4 G cell steps), so the step is kept to five
+  // instructions a cell, and the second level of the sums is touched only by runs long enough to use it.
   float4v acc[2][2], tot[2][2];
-  auto reset = [&]() {
+  bool folded = false;  // `tot` holds something
+  auto clear = [](float4v(&m)[2][2]) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
-        tot[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
-      }
+      for (int j = 0; j < 2; ++j) m[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
   };
-  auto adagrad = [&]() {  // AsyncAdagrad of one batch on the tile (async_adagrad.py:75-85)
+  auto gather_sums = [&]() {  // the run's gradient into `acc`
+    if (folded) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = tot[i][j] + acc[i][j];
+      clear(tot);
+      folded = false;
+    }
+  };
+  auto adagrad = [&]() {  // AsyncAdagrad of one batch on the tile (async_adagrad.py:75-85); the accumulators start over
+    gather_sums();
+    float least = INFINITY;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          // One such step per run and matrix cell is most of this kernel's arithmetic when the
-          // runs are short: the hardware's square root and reciprocal (1 ulp each) in place
-          // of the correctly rounded sequences.
-          const float g = tot[i][j][r] + acc[i][j][r];
-          const float sum = ht[i][j][r] + g * g;
+          const float sum = ht[i][j][r] + acc[i][j][r] * acc[i][j][r];
           ht[i][j][r] = sum;
-          wt[i][j][r] += -lr * g * __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(sum) + 1e-10f);
+          least = fminf(least, sum);
         }
+    // 1 / (sqrt(sum) + 1e-10): from sum = 2^-18 on the addition leaves sqrt(sum) as it is (1e-10 is below half its last
+    // digit), and the hardware's reciprocal square root (1 ulp) is the whole expression.
+    if (__any(least < 3.8147e-6f)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            wt[i][j][r] += -lr * acc[i][j][r] * __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(ht[i][j][r]) + 1e-10f);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) wt[i][j][r] += -lr * acc[i][j][r] * __builtin_amdgcn_rsqf(ht[i][j][r]);
+    }
+    clear(acc);
   };
-  reset();
+  clear(acc);
+  clear(tot);
 
   if (!RUNS && hot.part != nullptr) {
     const uint32_t slot = hot.hot_slot[rel];
@@ -447,10 +476,9 @@ __global__ __launch_bounds__(kThreads, 4) void seg_linear_update_kernel(
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) tot[i][j] += src[i * 2 + j];
+            for (int j = 0; j < 2; ++j) acc[i][j] += src[i * 2 + j];
         }
         adagrad();
-        reset();
       }
       write_back();
       return;
@@ -510,7 +538,6 @@ __global__ __launch_bounds__(kThreads, 4) void seg_linear_update_kernel(
       const uint32_t bt = (uint32_t)__builtin_amdgcn_readlane((int)mine, a);
       if (!RUNS && bt != cur) {  // (a part of a run is of one batch)
         if (cur != kNone) adagrad();
-        reset();
         steps = 0;
         cur = bt;
       }
@@ -527,6 +554,7 @@ __global__ __launch_bounds__(kThreads, 4) void seg_linear_update_kernel(
 #pragma unroll
           for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
         if ((++steps & (4 * kFoldTiles - 1)) == 0) {
+          folded = true;
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -548,10 +576,11 @@ __global__ __launch_bounds__(kThreads, 4) void seg_linear_update_kernel(
     __syncthreads();
   }
   if (RUNS) {
+    gather_sums();
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) part_out[i * 2 + j] = tot[i][j] + acc[i][j];
+      for (int j = 0; j < 2; ++j) part_out[i * 2 + j] = acc[i][j];
     return;
   }
   if (cur != kNone) adagrad();
