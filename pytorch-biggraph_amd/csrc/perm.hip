@@ -68,6 +68,122 @@ __global__ __launch_bounds__(256) void scatter_rows_multi_kernel(const uint4* __
   if (bad && v == 0 && oob_flag) *oob_flag = 1;
 }
 
+// ---- rows moved in place along the permutation's cycles ---------------------------------------
+// rows'[perm[i]] = rows[i] without a second table.  One position in every 16 is a leader (which one: a hash of the block, so
+// that no regular permutation avoids them); the leaders' rows are saved first.  A lane group then carries a leader's row
+// forward: read the row at perm[i], write the carried one there, go on with the one just read, until the next leader.  Every
+// row belongs to one such stretch, so nothing is read after another group wrote it.  Cycles without a leader (a handful of
+// short ones in a random permutation) are found by the marks the stretches left and moved by the wave that holds their
+// smallest position.
+// Bound by HBM: each row is read and written once, where scattering into a second table and copying it back reads and
+// writes it twice, and a row's write finds in L2 the lines that its read brought.  A stretch is a chain of dependent reads
+// (1 to 2 us a step), and the longest is what a small table waits for: stretches of 16 on average took 575 us for 1 GiB of 1 KiB
+// rows, of 32 712, of 32 with four to a lane group 740; the rows saved first cost a sixteenth of the traffic.
+// Permutation of 10.4 M rows of 400 bytes: 4.5 -> 3.2 ms.
+constexpr int kStretch = 16;
+constexpr int kLongestChain = 4096;  // a valid permutation exceeds this with probability n (15/16)^4096; an invalid one ends here
+
+__device__ __forceinline__ uint32_t leader_hash(uint64_t block) {
+  uint64_t x = block * 0x9e3779b97f4a7c15ull;
+  x ^= x >> 32;
+  x *= 0xd6e8feb86659fd93ull;
+  return (uint32_t)(x >> 40);
+}
+__device__ __forceinline__ int64_t leader_of(int64_t block) { return block * kStretch + (leader_hash((uint64_t)block) & (kStretch - 1)); }
+__device__ __forceinline__ bool is_leader(int64_t p) { return leader_of(p / kStretch) == p; }
+
+// saved[b] = the row of block b's leader; marks cleared.  One wave per block.
+__global__ __launch_bounds__(256) void cycle_save_kernel(const uint4* __restrict__ rows, int64_t n, int row_words,
+                                                         uint4* __restrict__ saved, uint8_t* __restrict__ mark) {
+  const int lane = threadIdx.x & 63;
+  const int64_t block = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (block * kStretch >= n) return;
+  if (lane < kStretch && block * kStretch + lane < n) mark[block * kStretch + lane] = 0;
+  const int64_t i = leader_of(block);
+  if (i >= n) return;
+  for (int v = lane; v < row_words; v += kWave) saved[block * row_words + v] = rows[i * row_words + v];
+}
+
+// LPR lanes carry a row, WPL 128-bit words each.
+template <int LPR, int WPL>
+__global__ __launch_bounds__(256) void cycle_walk_kernel(uint4* __restrict__ rows, int64_t n, int row_words,
+                                                         const int64_t* __restrict__ perm, const uint4* __restrict__ saved,
+                                                         uint8_t* __restrict__ mark, int32_t* __restrict__ oob_flag) {
+  constexpr int kGroups = 256 / LPR;
+  const int v = threadIdx.x % LPR;
+  const int64_t blocks = (n + kStretch - 1) / kStretch;
+  const int64_t block = (int64_t)blockIdx.x * kGroups + threadIdx.x / LPR;
+  if (block >= blocks) return;
+  const int64_t first = leader_of(block);
+  if (first >= n) return;
+  uint4 x[WPL];
+  int64_t p = perm[first];
+#pragma unroll
+  for (int w = 0; w < WPL; ++w) {
+    const int at = min(v + w * LPR, row_words - 1);
+    x[w] = saved[block * row_words + at];
+  }
+  for (int step = 0;; ++step) {
+    if (p < 0 || p >= n || step >= kLongestChain) {
+      if (v == 0 && oob_flag) *oob_flag = 1;
+      break;
+    }
+    uint4* row = rows + p * row_words;
+    const bool last = is_leader(p);
+    const int64_t next = perm[p];
+    uint4 y[WPL];
+#pragma unroll
+    for (int w = 0; w < WPL; ++w) y[w] = row[min(v + w * LPR, row_words - 1)];
+#pragma unroll
+    for (int w = 0; w < WPL; ++w)
+      if (v + w * LPR < row_words) row[v + w * LPR] = x[w];
+    if (last) break;
+    if (v == 0) mark[p] = 1;
+#pragma unroll
+    for (int w = 0; w < WPL; ++w) x[w] = y[w];
+    p = next;
+  }
+}
+
+// The cycles without a leader.
+template <int WPL>
+__global__ __launch_bounds__(256) void cycle_rest_kernel(uint4* __restrict__ rows, int64_t n, int row_words,
+                                                         const int64_t* __restrict__ perm, const uint8_t* __restrict__ mark,
+                                                         int32_t* __restrict__ oob_flag) {
+  const int lane = threadIdx.x & 63;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  bool least = false;  // i is the smallest position of such a cycle of two or more
+  if (i < n && !mark[i] && !is_leader(i)) {
+    int64_t p = perm[i];
+    for (int step = 0; p != i; ++step) {
+      if (p < 0 || p >= n || step >= kLongestChain) {
+        if (oob_flag) *oob_flag = 1;
+        break;
+      }
+      if (p < i || mark[p] || is_leader(p)) break;  // (of an invalid permutation: ran into another stretch)
+      p = perm[p];
+      least = p == i;
+    }
+  }
+  for (uint64_t todo = __ballot(least); todo != 0; todo &= todo - 1) {
+    const int64_t start = __shfl(i, __ffsll((unsigned long long)todo) - 1);
+    uint4 x[WPL];
+#pragma unroll
+    for (int w = 0; w < WPL; ++w) x[w] = rows[start * row_words + min(lane + w * kWave, row_words - 1)];
+    int64_t p = start;
+    do {  // (the cycle was walked above: it is closed)
+      p = perm[p];
+      uint4* row = rows + p * row_words;
+#pragma unroll
+      for (int w = 0; w < WPL; ++w) {
+        const uint4 y = row[min(lane + w * kWave, row_words - 1)];
+        if (lane + w * kWave < row_words) row[lane + w * kWave] = x[w];
+        x[w] = y;
+      }
+    } while (p != start);
+  }
+}
+
 // scalar rows (row = one 4- or 8-byte word): one thread per row
 template <typename WORD>
 __global__ void scatter_words_kernel(const WORD* __restrict__ rows, int64_t n, const int64_t* __restrict__ perm,
@@ -491,6 +607,36 @@ int scatter_rows(const void* rows, int64_t n, int64_t row_bytes, const int64_t* 
   }
   return check_launch("pbg_shuffle_rows");
 }
+
+// Whether moving rows along the cycles is the faster way (us, in place / through a second table): rows of 256 bytes 242 / 240
+// at 256 MiB, 687 / 863 at 1 GiB; of 400 bytes 263 / 279, 798 / 1093; of 1 KiB 194 / 230, 575 / 855; of 4 KiB 291 / 226, 769 / 838:
+// below, the second table stays in the memory-side cache.  Rows of 128 bytes gain nothing (956 / 871 at 1 GiB).
+bool cycles_pay(const void* rows, int64_t n, int64_t row_bytes, const void* scratch) {
+  const int64_t least = (int64_t)(row_bytes <= 1024 ? 512 : 1024) << 20;
+  return row_bytes % 16 == 0 && (uintptr_t)rows % 16 == 0 && (uintptr_t)scratch % 16 == 0 && row_bytes >= 256 && row_bytes <= 4096 &&
+         n * row_bytes >= least;
+}
+
+int shuffle_in_place(void* rows, int64_t n, int64_t row_bytes, const int64_t* perm, void* scratch, int32_t* oob_flag,
+                     hipStream_t s) {
+  const int words = (int)(row_bytes / 16);
+  const int64_t blocks = ceil_div(n, kStretch);
+  uint4* saved = (uint4*)scratch;
+  uint8_t* mark = (uint8_t*)scratch + blocks * row_bytes;  // (blocks rows and n bytes are less than n rows)
+  hipLaunchKernelGGL(cycle_save_kernel, dim3((unsigned)ceil_div(blocks, 4)), dim3(256), 0, s, (const uint4*)rows, n, words, saved, mark);
+  const auto walk = [&](auto kernel, int lpr) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(blocks, 256 / lpr)), dim3(256), 0, s, (uint4*)rows, n, words,
+                       perm, saved, mark, oob_flag);
+  };
+  if (words <= 16) walk(cycle_walk_kernel<16, 1>, 16);
+  else if (words <= 32) walk(cycle_walk_kernel<32, 1>, 32);
+  else if (words <= 64) walk(cycle_walk_kernel<64, 1>, 64);
+  else if (words <= 128) walk(cycle_walk_kernel<64, 2>, 64);
+  else walk(cycle_walk_kernel<64, 4>, 64);
+  const auto rest = words <= 64 ? cycle_rest_kernel<1> : words <= 128 ? cycle_rest_kernel<2> : cycle_rest_kernel<4>;
+  hipLaunchKernelGGL(rest, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, (uint4*)rows, n, words, perm, mark, oob_flag);
+  return check_launch("pbg_shuffle_rows");
+}
 }  // namespace
 
 extern "C" int pbg_shuffle_rows(void* rows, int64_t n, int64_t row_bytes, const int64_t* perm, void* scratch,
@@ -500,6 +646,7 @@ extern "C" int pbg_shuffle_rows(void* rows, int64_t n, int64_t row_bytes, const 
   if (!rows || !perm || !scratch) return fail(PBG_ERR_INVALID, "pbg_shuffle_rows: null pointer");
   if (row_bytes % 4 != 0) return fail(PBG_ERR_UNSUPPORTED, "pbg_shuffle_rows: row_bytes must be a multiple of 4");
   hipStream_t s = (hipStream_t)stream;
+  if (cycles_pay(rows, n, row_bytes, scratch)) return shuffle_in_place(rows, n, row_bytes, perm, scratch, oob_flag, s);
   // A valid permutation writes every scratch row; with an invalid one the flag
   // is raised and the contents of `rows` are unspecified (the reference throws
   // mid-way, util.cpp:200-202, leaving a partly shuffled tensor too).
