@@ -756,8 +756,10 @@ __global__ __launch_bounds__(kRowThreads) void ranks_out_kernel(StepCtx c, float
                                                                 float* __restrict__ rhs_pos,
                                                                 int64_t* __restrict__ lhs_rank,
                                                                 int64_t* __restrict__ rhs_rank,
-                                                                float* __restrict__ loss_edge) {
+                                                                float* __restrict__ loss_edge,
+                                                                unsigned long long* __restrict__ auc_hits) {
   const int lane = threadIdx.x & 63;
+  if (auc_hits && blockIdx.x == 0 && threadIdx.x < 2) auc_hits[threadIdx.x] = 0ull;  // auc_sample_kernel, behind this one, counts up
   const int64_t job = (int64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (job >= (int64_t)c.K * c.B) return;
   const int k = (int)(job / c.B), q = (int)(job % c.B);
@@ -814,10 +816,6 @@ __global__ __launch_bounds__(256) void auc_sample_kernel(StepCtx c, const float*
   }
   const uint64_t m = __ballot(hit);
   if ((threadIdx.x & 63) == 0 && m != 0ull) atomicAdd(&hits[s], (unsigned long long)__popcll(m));
-}
-
-__global__ void zero_u64_kernel(unsigned long long* p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -2891,10 +2889,9 @@ extern "C" int pbg_model_ranks(const pbg_step_desc* desc, const pbg_step_buffers
                          : longest <= 16 * kWave                            ? ranks_out_kernel<16>
                                                                             : ranks_out_kernel<32>;
   hipLaunchKernelGGL(ranks_out, wave_grid((int64_t)c.K * c.B), dim3(kRowThreads), 0, s, c, lhs_pos, rhs_pos, lhs_rank,
-                     rhs_rank, loss_edge);
+                     rhs_rank, loss_edge, auc_samples > 0 ? (unsigned long long*)auc_hits : nullptr);
   if (auc_samples > 0) {
     static_assert(sizeof(unsigned long long) == sizeof(int64_t), "auc_hits is written as two 64-bit counters");
-    hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, s, (unsigned long long*)auc_hits, 2);
     hipLaunchKernelGGL(auc_sample_kernel, dim3((unsigned)ceil_div(auc_samples, 256), 2), dim3(256), 0, s, c, lhs_pos, rhs_pos,
                        auc_samples, auc_seed, (unsigned long long*)auc_hits);
   }
@@ -2906,17 +2903,14 @@ namespace {
 // bytes per edge: bound by its launches (ten torch reductions, each read back by itself, took 300 microseconds for
 // the 10000 edges whose ranks take 400).
 constexpr int kRankSums = 14, kRankSumBlocks = 64;
-__device__ __forceinline__ double block_sum(double v, double* sh) {  // 256 threads
+__device__ __forceinline__ double wave_sum_double(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  return v;
 }
 __global__ __launch_bounds__(256) void rank_sums_kernel(IdArrays a, int64_t count, const int64_t* __restrict__ lhs_rank,
                                                         const int64_t* __restrict__ rhs_rank,
                                                         const float* __restrict__ loss_edge, double* __restrict__ partial) {
-  __shared__ double sh[4];
+  __shared__ double sh[4][kRankSums];
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, total = (int64_t)gridDim.x * 256;
   double v[kRankSums] = {};
   for (int64_t i = t; i < count; i += total) {
@@ -2935,19 +2929,23 @@ __global__ __launch_bounds__(256) void rank_sums_kernel(IdArrays a, int64_t coun
     if (ids_outside(a, which, t, total)) v[13] = 1.0;
 #pragma unroll
   for (int j = 0; j < kRankSums; ++j) {
-    const double sum = block_sum(v[j], sh);
-    if (threadIdx.x == 0) partial[(int64_t)blockIdx.x * kRankSums + j] = sum;
+    const double sum = wave_sum_double(v[j]);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][j] = sum;
   }
-}
-__global__ __launch_bounds__(64) void rank_sums_out_kernel(const double* __restrict__ partial, int blocks,
-                                                           const int64_t* __restrict__ auc_hits, double* __restrict__ out) {
+  __syncthreads();
   const int j = threadIdx.x;
-  if (j >= kRankSums) return;
-  double sum = 0.0;
-  for (int b = 0; b < blocks; ++b) sum += partial[(int64_t)b * kRankSums + j];
+  if (j < kRankSums) partial[(int64_t)blockIdx.x * kRankSums + j] = (sh[0][j] + sh[1][j]) + (sh[2][j] + sh[3][j]);
+}
+// Wave j adds up sum j of the (at most 64) blocks.
+static_assert(kRankSumBlocks <= kWave, "one block per lane");
+__global__ __launch_bounds__(kWave * kRankSums) void rank_sums_out_kernel(const double* __restrict__ partial, int blocks,
+                                                                          const int64_t* __restrict__ auc_hits,
+                                                                          double* __restrict__ out) {
+  const int j = threadIdx.x >> 6, b = threadIdx.x & 63;
+  double sum = wave_sum_double(b < blocks ? partial[(int64_t)b * kRankSums + j] : 0.0);
   if (j == 6) sum = auc_hits ? (double)auc_hits[0] : 0.0;
   if (j == 12) sum = auc_hits ? (double)auc_hits[1] : 0.0;
-  out[j] = sum;
+  if (b == 0) out[j] = sum;
 }
 }  // namespace
 
@@ -2968,7 +2966,7 @@ extern "C" int pbg_rank_sums(const pbg_step_desc* desc, const pbg_step_buffers* 
   if (blocks > kRankSumBlocks) blocks = kRankSumBlocks;
   hipLaunchKernelGGL(rank_sums_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, count, lhs_rank, rhs_rank,
                      loss_edge, (double*)scratch);
-  hipLaunchKernelGGL(rank_sums_out_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, (const double*)scratch, (int)blocks,
+  hipLaunchKernelGGL(rank_sums_out_kernel, dim3(1), dim3(kWave * kRankSums), 0, (hipStream_t)stream, (const double*)scratch, (int)blocks,
                      auc_hits, out);
   return check_launch("pbg_rank_sums");
 }
