@@ -17,6 +17,7 @@ struct SideCtx {
   int64_t num_rows;
   int all;              // RelationSchema.all_negs: the negatives are the table's rows 0 .. num_rows - 1 (u == num_rows)
   int nb, u, nn;        // batch-negative / uniform / total negative columns of this side
+  int ns;               // floats from one row of s (and of gs) to the next: nn, or more to start rows at cache lines
   int stride_p;         // rows per chunk of the buffer that holds the positives
   int alias;            // positives are the first P rows of the negatives matrix
   float *xn, *xp, *xa;  // prepared negatives matrix, positives, operated positives (dynamic)
@@ -25,7 +26,7 @@ struct SideCtx {
   float* bs;            // with config.bias: [K*C*P] row sums of dLoss/dscore of this side's score matrix
   float* gs;            // with config.bias and l2: [K*C, P, nn] dLoss/dscore itself (s then holds -2 dLoss/d squared distance, from which it cannot be read back)
   float *dxn, *dxp, *dxa;
-  float* s;             // [K*C, P, nn] scores against this side's negatives, then dLoss/dS
+  float* s;             // [K*C, P, ns] scores against this side's negatives, then dLoss/dS
   float* rs;            // [K*C*P] row sums of dLoss/d(squared distance) (l2)
   int slot_pos, slot_uni;
   // The gradient rows of this side's uniform negatives are read where the backward GEMM wrote them
