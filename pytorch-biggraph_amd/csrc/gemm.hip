@@ -328,24 +328,45 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_kernel(GemmArgs g, int t
       return;
     }
   }
+  auto store = [&](int i, int j, int r, auto&& finish) {
+    const int col = n0 + wn0 + j * 16 + (lane & 15);
+    const int row = m0 + wm0 + i * 16 + 4 * (lane >> 4) + r;
+    if (row < g.m && col < g.n) {
+      const float v = finish(g.alpha * (tot[i][j][r] + acc[i][j][r]));
+      c[(int64_t)row * g.ldc + col] = HALF ? (float)(_Float16)v : v;
+    }
+  };
+  if (g.beta == 0.f) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) store(i, j, r, [](float v) { return v; });
+    return;
+  }
+  // What is there already is read a row of tiles ahead of its use, from clamped addresses: a read behind each store (which it
+  // might alias) made 64 round trips of the epilogue, 25 us of a workgroup's 115 (80 products of 1000 x 1024 x 1100: 1.18 -> 1.03 ms;
+  // float16 0.69 -> 0.51).
+  float old[2][TN][4];
+  auto read_old = [&](int i, float(&o)[TN][4]) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[j][r] = c[(int64_t)min(m0 + wm0 + i * 16 + 4 * (lane >> 4) + r, g.m - 1) * g.ldc + min(n0 + wn0 + j * 16 + (lane & 15), g.n - 1)];
+  };
+  read_old(0, old[0]);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
+    if (i + 1 < TM) read_old(i + 1, old[(i + 1) & 1]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = n0 + wn0 + j * 16 + (lane & 15);
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm0 + i * 16 + 4 * (lane >> 4) + r;
-        if (row < g.m && col < g.n) {
-          float* dst = c + (int64_t)row * g.ldc + col;
-          float v = g.alpha * (tot[i][j][r] + acc[i][j][r]);
-          // HALF: the product is a Half tensor of its own before autograd adds it to what is there
-          // (two roundings: of the product, then of the sum)
-          if (g.beta != 0.f) v = (HALF ? (float)(_Float16)v : v) + g.beta * *dst;
-          *dst = HALF ? (float)(_Float16)v : v;
-        }
-      }
-    }
+      for (int r = 0; r < 4; ++r)
+        // HALF: the product is a Half tensor of its own before autograd adds it to what is there
+        // (two roundings: of the product, then of the sum)
+        store(i, j, r, [&](float v) { return (HALF ? (float)(_Float16)v : v) + g.beta * old[i & 1][j][r]; });
   }
 }
 
