@@ -1,4 +1,4 @@
-"""`linear` with one relation per edge at the edges of its kernels' tiles (64 sorted edges x 128 columns, 32 values of k):
+"""`linear` with one relation per edge at the edges of its kernels' tiles (64 sorted edges x 64 columns, 16 values of k):
 both directions of the per-relation products against the oracle, dims that no vector load fits among them, and tiles that
 hold one relation, several, or part of one.  Criterion and slack are those of the many-workers comparison (Adagrad turns a
 gradient that is rounding noise into a full step)."""
