@@ -377,14 +377,16 @@ int pbg_reverse_permutation(const int64_t* perm, int64_t n, int64_t* out, pbg_st
 
 /* _C.shuffle (util.cpp:127-220): rows[perm[i]] <- rows[i], result left in
  * `rows`.  `scratch` holds n * row_bytes bytes.  row_bytes must be a multiple
- * of 4.  An out-of-range perm entry sets *oob_flag and drops that row. */
+ * of 4.  An out-of-range perm entry sets *oob_flag; the contents of `rows`
+ * are then unspecified, as they are where perm names a row twice.  Large
+ * tables are moved in place and touch a sixteenth of `scratch`. */
 int pbg_shuffle_rows(void* rows, int64_t n, int64_t row_bytes, const int64_t* perm, void* scratch,
                      int32_t* oob_flag, pbg_stream_t stream);
 
 /* The same move out of place: out[perm[i]] <- rows[i], `rows` untouched, `out`
  * (n * row_bytes bytes) not overlapping it.  For a caller that holds two
- * buffers and swaps them, so that the copy back of the in-place form (half of
- * its traffic) is not paid.  The reference only has the in-place form
+ * buffers and swaps them: no copy back (small tables, narrow or very wide rows
+ * above) and no chains of dependent reads.  The reference only has the in-place form
  * (util.cpp:127-220, whose cycle-following needs no second buffer on a CPU). */
 int pbg_shuffle_rows_out(const void* rows, int64_t n, int64_t row_bytes, const int64_t* perm, void* out,
                          int32_t* oob_flag, pbg_stream_t stream);
